@@ -139,6 +139,9 @@ def lib() -> C.CDLL:
                  "mmm_contract5d_truth_f64", "mmm_gemm_plan_f16f32", "mmm_probe_clock", "mmm_probe_mfma_ceiling",
                  "mmm_probe_lds_mfma", "mmm_probe_read"):
         getattr(L, name).restype = C.c_int
+    # of the HIP runtime the library is bound to
+    L.hipStreamGetCaptureInfo.argtypes = [s, C.POINTER(i), C.POINTER(C.c_ulonglong)]
+    L.hipStreamGetCaptureInfo.restype = C.c_int
     L.mmm_version.restype = C.c_char_p
     L.mmm_version.argtypes = []
     _lib = L
@@ -177,12 +180,57 @@ TILES = {"256x256": (4, 4, 2, 2), "128x256": (2, 4, 2, 2), "256x128": (4, 2, 2, 
 MAX_WORKSPACE_BYTES = 64 << 20
 
 # K-split workspaces the wrappers pass to the library: one per (device, stream), from torch's
-# allocator, grown on demand.  Calls on one stream are ordered, so they may share one, but a call
+# allocator, grown on demand; calls captured into a graph get one of the graph's own
+# (_graph_workspace).  Calls on one stream are ordered, so they may share one, but a call
 # that splits K is two launches: _launch_lock keeps them together when several host threads call on
 # one stream (the second thread's partial sums must not land between the first's two launches).
 _ws_lock = threading.Lock()
 _launch_lock = threading.Lock()
 _ws_cache = {}
+_graph_pool = (None, False)  # the last capture seen, and whether torch allocates for it from a pool of its own
+
+
+def _capture_id(st: C.c_void_p):
+    """The id of the graph capture that stream `st` is part of, or None (the null stream cannot be)."""
+    if not st.value:
+        return None
+    status, ident = C.c_int(), C.c_ulonglong()
+    rc = lib().hipStreamGetCaptureInfo(st, C.byref(status), C.byref(ident))
+    return ident.value if rc == HIP_SUCCESS and status.value == 1 else None
+
+
+def _graph_workspace(device, st: C.c_void_p, capture: int, nbytes: int):
+    """A workspace for one call captured on `st`.  A graph replays on any stream, beside other graphs
+    captured on the same one and beside eager calls, so it cannot use the per-stream workspace: it
+    gets memory from the pool that torch keeps for the graph as long as the graph lives.  The tensor
+    may go when the call returns: the pool gives its memory only to later work of the same stream in
+    the same graph.  None (unsplit kernels) if the capture is not torch's: its memory would be reused."""
+    import torch
+
+    global _graph_pool
+    with torch.cuda.stream(torch.cuda.ExternalStream(st.value, device=device)):
+        t = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    seen, private = _graph_pool
+    if seen != capture:  # one snapshot a capture
+        at = t.data_ptr()
+        private = any(g["address"] <= at < g["address"] + g["total_size"] and tuple(g["segment_pool_id"]) != (0, 0)
+                      for g in torch.cuda.memory_snapshot())
+        _graph_pool = (capture, private)
+    return t if private else None
+
+
+def _gemm_need(A, B, C_out, M, N, K, lda, ldb, ldc) -> int:
+    n = C.c_size_t()
+    _check("mmm_gemm_workspace_f16f32",
+           lib().mmm_gemm_workspace_f16f32(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, C.byref(n)))
+    return n.value
+
+
+def _contract_need(desc, A, B, C_out) -> int:
+    n = C.c_size_t()
+    _check("mmm_contract5d_workspace_f16f32",
+           lib().mmm_contract5d_workspace_f16f32(C.byref(desc), _ptr(A), _ptr(B), _ptr(C_out), C.byref(n)))
+    return n.value
 
 
 def _workspace(device, st: C.c_void_p, nbytes: int):
@@ -197,13 +245,25 @@ def _workspace(device, st: C.c_void_p, nbytes: int):
         return t
 
 
-def _ws_args(workspace, device, st, nbytes: int):
-    """(pointer, bytes) for a call needing nbytes: the caller's tensor, none (workspace=False),
-    or the per-stream cache."""
-    if workspace is False or nbytes == 0:
-        return None, 0
-    t = workspace if workspace is not None else _workspace(device, st, nbytes)
-    return C.c_void_p(t.data_ptr()), t.numel() * t.element_size()
+def _ws_of(t):
+    return (None, 0) if t is None else (C.c_void_p(t.data_ptr()), t.numel() * t.element_size())
+
+
+def _ws_args(workspace, device, st, need):
+    """(tensor, pointer, bytes) for a call: the caller's tensor, none (workspace=False), the per-stream
+    cache's, or under graph capture one of need() bytes of the graph's own (at least 16: with a
+    workspace the library may choose another unsplit kernel than without).  The caller keeps the
+    tensor until its launch has been enqueued."""
+    if workspace is False:
+        return None, None, 0
+    t = workspace
+    if t is None:
+        capture = _capture_id(st)
+        if capture is None:
+            t = _workspace(device, st, MAX_WORKSPACE_BYTES)
+        else:
+            t = _graph_workspace(device, st, capture, max(need(), 16))
+    return t, *_ws_of(t)
 
 
 def gemm(A, B, C_out=None, tile=None, stream=None, workspace=None):
@@ -235,24 +295,17 @@ def gemm(A, B, C_out=None, tile=None, stream=None, workspace=None):
     L = lib()
     if tile is None:
         # one library call: the per-stream workspace holds the largest split the library plans
-        wp, wb = _ws_args(workspace, A.device, st, MAX_WORKSPACE_BYTES)
+        ws, wp, wb = _ws_args(workspace, A.device, st, lambda: _gemm_need(A, B, C_out, M, N, K, lda, ldb, ldc))
         with _launch_lock:
             rc = L.mmm_gemm_f16f32_ws(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, wp, wb, st)
         _check("mmm_gemm_f16f32_ws", rc)
     else:
         params = TILES[tile] if isinstance(tile, str) else tuple(tile)
-        wp, wb = _ws_args(workspace, A.device, st, MAX_WORKSPACE_BYTES)
+        ws, wp, wb = _ws_args(workspace, A.device, st, lambda: MAX_WORKSPACE_BYTES)
         with _launch_lock:
             rc = L.mmm_gemm_f16f32_tiled(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, *params, wp, wb, st)
         _check("mmm_gemm_f16f32_tiled", rc)
     return C_out
-
-
-def _ws_tensor(workspace, device, st):
-    """The workspace tensor a bound launcher keeps alive: the caller's, the per-stream one, or None."""
-    if workspace is False:
-        return None
-    return workspace if workspace is not None else _workspace(device, st, MAX_WORKSPACE_BYTES)
 
 
 def _bound(fn, name: str, args: tuple, keep: tuple):
@@ -263,6 +316,42 @@ def _bound(fn, name: str, args: tuple, keep: tuple):
             raise MMMError(name, rc)
 
     launch.tensors = keep  # the launcher holds its operands (and workspace) alive
+    return launch
+
+
+def _bound_ws(fn, name: str, args, workspace, device, st, need, keep: tuple):
+    """As _bound, for a call that takes a workspace: args(pointer, bytes) is the whole argument list.
+    With the default workspace the eager launches share the per-stream one, and a launch under graph
+    capture takes one of the graph's own."""
+    if workspace is not None or not st.value:  # fixed, or the null stream, which no graph captures
+        ws = None if workspace is False else workspace if workspace is not None else \
+            _workspace(device, st, MAX_WORKSPACE_BYTES)
+        return _bound(fn, name, args(*_ws_of(ws)), keep + (ws,))
+    eager = None
+
+    def bind_eager():
+        nonlocal eager
+        ws = _workspace(device, st, MAX_WORKSPACE_BYTES)
+        eager = args(*_ws_of(ws))
+        launch.tensors = keep + (ws,)
+
+    def launch():
+        capture = _capture_id(st)
+        if capture is not None:
+            ws = _graph_workspace(device, st, capture, max(need(), 16))
+            call = args(*_ws_of(ws))
+        else:
+            if eager is None:
+                bind_eager()
+            call = eager
+        with _launch_lock:
+            rc = fn(*call)
+        if rc != HIP_SUCCESS:
+            raise MMMError(name, rc)
+
+    launch.tensors = keep
+    if _capture_id(st) is None:  # a tensor made under capture would be the graph's
+        bind_eager()
     return launch
 
 
@@ -279,15 +368,14 @@ def bind_gemm(A, B, C_out, stream=None, workspace=None, tile=None):
         raise ValueError("C must be a row-major float32 [M,N] tensor")
     M, N, K, lda, ldb, ldc = _gemm_shapes(A, B, C_out)
     st = _stream(stream)
-    ws = _ws_tensor(workspace, A.device, st)
-    wp = C.c_void_p(ws.data_ptr()) if ws is not None else None
-    wb = ws.numel() * ws.element_size() if ws is not None else 0
+    head = (_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc)
     if tile is not None:
         params = TILES[tile] if isinstance(tile, str) else tuple(tile)
-        args = (_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, *params, wp, wb, st)
-        return _bound(lib().mmm_gemm_f16f32_tiled, "mmm_gemm_f16f32_tiled", args, (A, B, C_out, ws))
-    args = (_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, wp, wb, st)
-    return _bound(lib().mmm_gemm_f16f32_ws, "mmm_gemm_f16f32_ws", args, (A, B, C_out, ws))
+        return _bound_ws(lib().mmm_gemm_f16f32_tiled, "mmm_gemm_f16f32_tiled",
+                         lambda wp, wb: (*head, *params, wp, wb, st), workspace, A.device, st,
+                         lambda: MAX_WORKSPACE_BYTES, (A, B, C_out))
+    return _bound_ws(lib().mmm_gemm_f16f32_ws, "mmm_gemm_f16f32_ws", lambda wp, wb: (*head, wp, wb, st), workspace,
+                     A.device, st, lambda: _gemm_need(A, B, C_out, M, N, K, lda, ldb, ldc), (A, B, C_out))
 
 
 def bind_gemm_clocked(A, B, C_out, clock, stream=None, workspace=None):
@@ -301,23 +389,17 @@ def bind_gemm_clocked(A, B, C_out, clock, stream=None, workspace=None):
         raise ValueError("clock must be a contiguous CUDA int64 tensor [n, 4]")
     M, N, K, lda, ldb, ldc = _gemm_shapes(A, B, C_out)
     st = _stream(stream)
-    ws = _ws_tensor(workspace, A.device, st)
-    wp = C.c_void_p(ws.data_ptr()) if ws is not None else None
-    wb = ws.numel() * ws.element_size() if ws is not None else 0
-    fn = lib().mmm_gemm_f16f32_clocked
+    clocked = lib().mmm_gemm_f16f32_clocked
     state = {"i": 0}
-    base = (_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, wp, wb)
 
-    def launch():
+    def fn(*args):
         slot = C.c_void_p(clock.data_ptr() + 32 * (state["i"] % clock.shape[0]))
         state["i"] += 1
-        with _launch_lock:
-            rc = fn(*base, slot, st)
-        if rc != HIP_SUCCESS:
-            raise MMMError("mmm_gemm_f16f32_clocked", rc)
+        return clocked(*args, slot, st)
 
-    launch.tensors = (A, B, C_out, ws, clock)
-    return launch
+    head = (_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc)
+    return _bound_ws(fn, "mmm_gemm_f16f32_clocked", lambda wp, wb: (*head, wp, wb), workspace, A.device, st,
+                     lambda: _gemm_need(A, B, C_out, M, N, K, lda, ldb, ldc), (A, B, C_out, clock))
 
 
 def clocks_mhz(clock):
@@ -337,11 +419,9 @@ def bind_contract(desc: "ContractDesc", A, B, C_out, stream=None, workspace=None
         raise TypeError("C must be a CUDA float32 tensor")
     st = _stream(stream)
     d = ContractDesc.from_buffer_copy(desc)
-    ws = _ws_tensor(workspace, A.device, st)
-    wp = C.c_void_p(ws.data_ptr()) if ws is not None else None
-    wb = ws.numel() * ws.element_size() if ws is not None else 0
-    args = (C.pointer(d), _ptr(A), _ptr(B), _ptr(C_out), wp, wb, st)
-    return _bound(lib().mmm_contract5d_f16f32_ws, "mmm_contract5d_f16f32_ws", args, (A, B, C_out, ws, d))
+    return _bound_ws(lib().mmm_contract5d_f16f32_ws, "mmm_contract5d_f16f32_ws",
+                     lambda wp, wb: (C.pointer(d), _ptr(A), _ptr(B), _ptr(C_out), wp, wb, st), workspace, A.device, st,
+                     lambda: _contract_need(d, A, B, C_out), (A, B, C_out, d))
 
 
 KERNELS = {0: "none", 1: "zero", 2: "tile", 3: "stream", 4: "tile+stream"}
@@ -442,7 +522,7 @@ def contract(desc: ContractDesc, A, B, C_out, stream=None, workspace=None):
         raise TypeError("C must be a CUDA float32 tensor")
     st = _stream(stream)
     L = lib()
-    wp, wb = _ws_args(workspace, A.device, st, MAX_WORKSPACE_BYTES)
+    ws, wp, wb = _ws_args(workspace, A.device, st, lambda: _contract_need(desc, A, B, C_out))
     with _launch_lock:
         rc = L.mmm_contract5d_f16f32_ws(C.byref(desc), _ptr(A), _ptr(B), _ptr(C_out), wp, wb, st)
     _check("mmm_contract5d_f16f32_ws", rc)

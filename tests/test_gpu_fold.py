@@ -184,6 +184,46 @@ def test_fold_splits_threads_one_stream(mm, cuda):
     assert not wrong, wrong
 
 
+@pytest.mark.parametrize("bound", [False, True], ids=["contract", "bind_contract"])
+def test_fold_split_graphs_at_once(mm, cuda, bound, monkeypatch):
+    """Split contractions captured into two graphs on one stream, replayed at the same time on two
+    others beside eager calls on the stream of the capture: each has partial sums of its own."""
+    cases = [_check(cuda, mm, (8, 256, 1, 16, 40, 128), KM, seed=s) for s in range(3)]
+    side, graphs, own = cuda.cuda.Stream(), [], []
+    take = mm._graph_workspace
+
+    def spy(*args):
+        t = take(*args)
+        own.append((len(graphs), t.data_ptr(), t.numel()))
+        return t
+
+    monkeypatch.setattr(mm, "_graph_workspace", spy)
+    side.wait_stream(cuda.cuda.current_stream())
+    for d, A, B, C, T in cases[:2]:
+        g = cuda.cuda.CUDAGraph()
+        launch = mm.bind_contract(d, A, B, C, stream=side) if bound else lambda: mm.contract(d, A, B, C)
+        with cuda.cuda.graph(g, stream=side):
+            launch()
+            launch()
+        graphs.append(g)
+    assert [g for g, _, _ in own] == [0, 0, 1, 1] and all(n > 16 for _, _, n in own)
+    assert not {p for g, p, _ in own if g == 0} & {p for g, p, _ in own if g == 1}
+    streams = [cuda.cuda.Stream(), cuda.cuda.Stream()]
+    d, A, B, C, T = cases[2]
+    for i in range(10):
+        for c in cases:
+            c[3].fill_(float("nan"))
+        cuda.cuda.synchronize()
+        for s, g in zip(streams, graphs):
+            with cuda.cuda.stream(s):
+                g.replay()
+        with cuda.cuda.stream(side):
+            mm.contract(d, A, B, C)
+        cuda.cuda.synchronize()
+        for j, c in enumerate(cases):
+            assert cuda.equal(c[3], c[4]), f"pass {i}: contraction {j}"
+
+
 # 33 to 64 rows of a row-major GEMM on the fold kernel's skinny tiles: one K tile and K ends inside one,
 # odd K and N, a last strip of one column, rows at 2-byte alignment, 256-column strips, one strip, B from
 # 96 MiB (non-temporal); the view's padding is NaN

@@ -452,3 +452,40 @@ def test_contract_workspace_query(mm):
     assert 0 < need(128, 16, 64, 64, 128) <= mm.MAX_WORKSPACE_BYTES
     assert need(128, 8192, 64, 64, 128) == 0
     assert need(128, 16, 64, 1, 64) == 0
+
+
+def test_captured_calls_get_their_own_workspace(mm, monkeypatch):
+    """A graph replays beside others captured on the same stream, so a captured call's partial sums go
+    to memory of the graph's pool, not to the stream's shared workspace (host logic; no GPU)."""
+    import contextlib
+
+    import torch
+
+    dev, st = torch.device("cpu"), C.c_void_p(0x40)
+    pool = [(0, 1)]
+    monkeypatch.setattr(mm, "_capture_id", lambda s: 11)
+    monkeypatch.setattr(mm, "_graph_pool", (None, False))
+    monkeypatch.setattr(mm, "_ws_cache", {})
+    monkeypatch.setattr(torch.cuda, "ExternalStream", lambda *a, **k: None)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "memory_snapshot",
+                        lambda: [{"address": 0, "total_size": 1 << 62, "segment_pool_id": pool[0]}])
+    a, pa, na = mm._ws_args(None, dev, st, lambda: 4096)
+    b, pb, nb = mm._ws_args(None, dev, st, lambda: 0)
+    assert na == 4096 and nb == 16 and pa.value == a.data_ptr() != pb.value and not mm._ws_cache
+    own = torch.empty(64, dtype=torch.uint8)
+    assert mm._ws_args(own, dev, st, None)[1].value == own.data_ptr()
+    assert mm._ws_args(False, dev, st, None) == (None, None, 0)
+
+    seen = []
+    launch = mm._bound_ws(lambda *x: seen.append(x) or 0, "f", lambda wp, wb: (wp, wb), None, dev, st, lambda: 512, ())
+    launch()
+    assert seen[0][1] == 512 and not mm._ws_cache  # bound and launched under capture
+    monkeypatch.setattr(mm, "_capture_id", lambda s: None)
+    monkeypatch.setattr(mm, "_workspace", lambda *x: own)
+    launch()
+    assert seen[1][0].value == own.data_ptr()  # the same launcher, eager again
+    # a capture that torch does not allocate for: nothing would keep the memory, so no split
+    pool[0] = (0, 0)
+    monkeypatch.setattr(mm, "_capture_id", lambda s: 12)
+    assert mm._ws_args(None, dev, st, lambda: 4096) == (None, None, 0)
