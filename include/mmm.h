@@ -30,11 +30,14 @@
  *    M == 0 or N == 0 is a no-op; K == 0 writes zeros to C.
  *  - Work is enqueued on `stream` (0 = the null stream, as the reference) and is
  *    asynchronous, as the reference's launches are (the caller synchronises, mmm.cpp:1491).
- *  - Thread safety: the only mutable global state is mmm_gemm_f16f32_noalloc's: its 64 MiB
+ *  - Thread safety: the mutable global state is mmm_gemm_f16f32_noalloc's -- its 64 MiB
  *    device array (shared by every call of that entry point on one GPU) and a mutex-guarded
- *    table of the array's device address per GPU, filled on the first call on each GPU.  A
- *    workspace serves one call at a time: calls on one stream may share one (they are
- *    ordered); concurrent calls on different streams need their own.
+ *    table of the array's device address per GPU, filled on the first call on each GPU -- and a
+ *    mutex-guarded list of the streams on which a call that splits K is being launched.  A
+ *    workspace serves one call at a time: calls on one stream may share one, also from several
+ *    host threads (they are ordered, and the two launches of a split call are kept together:
+ *    a second thread's split call on that stream waits until both are enqueued); concurrent
+ *    calls on different streams, and graphs that may replay at the same time, need their own.
  */
 #ifndef MMM_H
 #define MMM_H

@@ -184,6 +184,43 @@ def test_fold_splits_threads_one_stream(mm, cuda):
     assert not wrong, wrong
 
 
+def test_split_entry_points_threads_one_stream(mm, cuda):
+    """The C entry points from several host threads on one stream with one workspace, as the header
+    allows: a fold, the streaming kernels' splits and a tile split, each with its own values."""
+    import ctypes as C
+    import threading
+
+    L, ws, st = mm.lib(), cuda.empty(mm.MAX_WORKSPACE_BYTES, dtype=cuda.uint8, device="cuda"), None
+    ptr = lambda t: C.c_void_p(t.data_ptr())
+    calls = []
+    for s in range(2):
+        d, A, B, Cd, T = _check(cuda, mm, (8, 256, 1, 16, 20, 128), KM, seed=s)
+        calls.append((L.mmm_contract5d_f16f32_ws, (C.byref(d), ptr(A), ptr(B), ptr(Cd), ptr(ws), ws.numel(), st), Cd, T,
+                      (d, A, B)))
+    for M, N, K in ((16, 4096, 4096), (40, 2048, 4096), (256, 256, 8192)):
+        gen = cuda.Generator(device="cuda").manual_seed(M)
+        A, B = (cuda.randint(-4, 5, x, generator=gen, device="cuda").half() for x in ((M, K), (K, N)))
+        Cd, T = cuda.empty(M, N, device="cuda"), (A.double() @ B.double()).float()
+        assert mm.gemm_plan(M, N, K)["workspace_bytes"] > 0
+        calls.append((L.mmm_gemm_f16f32_ws, (ptr(A), ptr(B), ptr(Cd), M, N, K, K, N, N, ptr(ws), ws.numel(), st), Cd, T,
+                      (A, B)))
+    cuda.cuda.synchronize()
+    wrong = []
+
+    def work(i, fn, args, Cd, T, keep):
+        rc = [fn(*args) for _ in range(200)]
+        cuda.cuda.synchronize()
+        if any(rc) or not cuda.equal(Cd, T):
+            wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i, *c)) for i, c in enumerate(calls)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong
+
+
 @pytest.mark.parametrize("bound", [False, True], ids=["contract", "bind_contract"])
 def test_fold_split_graphs_at_once(mm, cuda, bound, monkeypatch):
     """Split contractions captured into two graphs on one stream, replayed at the same time on two
