@@ -181,11 +181,9 @@ MAX_WORKSPACE_BYTES = 64 << 20
 
 # K-split workspaces the wrappers pass to the library: one per (device, stream), from torch's
 # allocator, grown on demand; calls captured into a graph get one of the graph's own
-# (_graph_workspace).  Calls on one stream are ordered, so they may share one, but a call
-# that splits K is two launches: _launch_lock keeps them together when several host threads call on
-# one stream (the second thread's partial sums must not land between the first's two launches).
+# (_graph_workspace).  Calls on one stream are ordered, so they may share one, also when several host
+# threads make them: the library keeps the two launches of a call that splits K together.
 _ws_lock = threading.Lock()
-_launch_lock = threading.Lock()
 _ws_cache = {}
 _graph_pool = (None, False)  # the last capture seen, and whether torch allocates for it from a pool of its own
 
@@ -296,22 +294,19 @@ def gemm(A, B, C_out=None, tile=None, stream=None, workspace=None):
     if tile is None:
         # one library call: the per-stream workspace holds the largest split the library plans
         ws, wp, wb = _ws_args(workspace, A.device, st, lambda: _gemm_need(A, B, C_out, M, N, K, lda, ldb, ldc))
-        with _launch_lock:
-            rc = L.mmm_gemm_f16f32_ws(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, wp, wb, st)
+        rc = L.mmm_gemm_f16f32_ws(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, wp, wb, st)
         _check("mmm_gemm_f16f32_ws", rc)
     else:
         params = TILES[tile] if isinstance(tile, str) else tuple(tile)
         ws, wp, wb = _ws_args(workspace, A.device, st, lambda: MAX_WORKSPACE_BYTES)
-        with _launch_lock:
-            rc = L.mmm_gemm_f16f32_tiled(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, *params, wp, wb, st)
+        rc = L.mmm_gemm_f16f32_tiled(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, *params, wp, wb, st)
         _check("mmm_gemm_f16f32_tiled", rc)
     return C_out
 
 
 def _bound(fn, name: str, args: tuple, keep: tuple):
     def launch():
-        with _launch_lock:
-            rc = fn(*args)
+        rc = fn(*args)
         if rc != HIP_SUCCESS:
             raise MMMError(name, rc)
 
@@ -344,8 +339,7 @@ def _bound_ws(fn, name: str, args, workspace, device, st, need, keep: tuple):
             if eager is None:
                 bind_eager()
             call = eager
-        with _launch_lock:
-            rc = fn(*call)
+        rc = fn(*call)
         if rc != HIP_SUCCESS:
             raise MMMError(name, rc)
 
@@ -523,8 +517,7 @@ def contract(desc: ContractDesc, A, B, C_out, stream=None, workspace=None):
     st = _stream(stream)
     L = lib()
     ws, wp, wb = _ws_args(workspace, A.device, st, lambda: _contract_need(desc, A, B, C_out))
-    with _launch_lock:
-        rc = L.mmm_contract5d_f16f32_ws(C.byref(desc), _ptr(A), _ptr(B), _ptr(C_out), wp, wb, st)
+    rc = L.mmm_contract5d_f16f32_ws(C.byref(desc), _ptr(A), _ptr(B), _ptr(C_out), wp, wb, st)
     _check("mmm_contract5d_f16f32_ws", rc)
     return C_out
 

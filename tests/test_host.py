@@ -551,3 +551,25 @@ int main() {
         text = open(os.path.join(csrc, name)).read()
         at = text.index("hipLaunchKernelGGL((" + launches)
         assert "StreamPair pair(" in text[text.rindex("static hipError_t ", 0, at):at], name
+
+
+def test_launches_do_not_wait_for_each_other(mm, monkeypatch):
+    """A launch that blocks (its stream's queue is full) holds up no other thread's launch (host logic)."""
+    import threading
+
+    blocked, release, through = threading.Event(), threading.Event(), threading.Event()
+
+    def slow():
+        blocked.set()
+        return 0 if release.wait(60) else 1
+
+    one = threading.Thread(target=mm._bound(slow, "slow", (), ()), daemon=True)
+    two = threading.Thread(target=mm._bound(lambda: through.set() or 0, "quick", (), ()), daemon=True)
+    one.start()
+    assert blocked.wait(30)
+    two.start()
+    passed = through.wait(10)
+    release.set()
+    one.join(60)
+    two.join(60)
+    assert passed
