@@ -407,6 +407,8 @@ __device__ __forceinline__ void ktile_last_step(const char LDS_AS* ns, const uin
 // tail_patch(slot) runs once this wave's loads of the last tile (in ring slot `slot`) have
 // landed, before the barrier that publishes it: a thread may overwrite the chunks its own
 // loads put there.  tile_patch(t, slot) is the same for every tile t, called before tail_patch.
+// tile_done(t) runs when the MFMAs of tile t (not the last) have been issued; half_done() before the
+// last K-step of each tile of a loop of at most S + 1 tiles, and of the last S + 1 of a longer one.
 struct NoHook {
   __device__ __forceinline__ void operator()() const {}
 };
@@ -416,13 +418,14 @@ struct NoSlotHook {
 };
 
 template <class T, bool BKM, int NST = 0, class Prep, class DmaOne, class IssueTile, class FirstWait = NoHook,
-          class TailPatch = NoSlotHook, class TilePatch = NoSlotHook, class TileDone = NoSlotHook>
+          class TailPatch = NoSlotHook, class TilePatch = NoSlotHook, class TileDone = NoSlotHook,
+          class HalfDone = NoHook>
 __device__ __forceinline__ void cross_stage(char LDS_AS* lds_base, int KT, bool tail_regs, const uint32_t (&a_off)[kMaxOff],
                                             const uint32_t (&b_off)[kMaxOff], AccT<T> (&acc)[T::FM][T::FN], Prep&& prep,
                                             DmaOne&& dma_one, IssueTile&& issue_tile, int pre = 0,
                                             FirstWait&& first_wait = FirstWait{}, TailPatch&& tail_patch = TailPatch{},
                                             TilePatch&& tile_patch = TilePatch{},
-                                            TileDone&& tile_done = TileDone{}) {
+                                            TileDone&& tile_done = TileDone{}, HalfDone&& half_done = HalfDone{}) {
   // Ring of S slots, tile u in slot u % S.  Cross-stage pipeline: during the last K-step of
   // tile t, this wave waits for its own loads of tile t+1, then the barrier (a) publishes
   // tile t+1 -- every wave's loads of it have landed -- and (b) retires slot t % S: every
@@ -492,16 +495,19 @@ __device__ __forceinline__ void cross_stage(char LDS_AS* lds_base, int KT, bool 
   }
   if (t + S == KT - 1) {
     tile_body();
+    half_done();
     tile_next(t, [&] { issue_tile(t + S, cur); });
     tile_done(t);
     ++t;
   }
   for (; t + 1 < KT; ++t) {
     tile_body();
+    half_done();
     tile_next(t, [] {});
     tile_done(t);
   }
   tile_body();
+  half_done();
   mfma_frags<T>(f[1], acc);
 }
 

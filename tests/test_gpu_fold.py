@@ -299,3 +299,40 @@ def test_gemm_33_to_64_rows_rounding(mm, cuda, shape):
     print(f"[gemm 33-64 rows] rounding {shape}", flush=True)
     T = A.double() @ B.double()
     assert ((mm.gemm(A, B) - T).norm() / T.norm()).item() <= 2e-7
+
+
+@pytest.mark.parametrize("k", [64, 96, 128])
+def test_gemm_33_to_64_rows_rounding_short(mm, cuda, k):
+    """Up to seven 32-row K steps: a chain of MFMAs per step.  There is a rounding per 8 products, of partial
+    sums of 8, 16, 24 and 32 products in each chain, then of the chains' sums.  A partial sum of s products
+    of operands uniform in [-1, 1) is near N(0, s / 9), its rounding uniform in half an ulp either way:
+    that gives the distance from fp64 up to a constant of the matrix cores' own, which K = 32 (one chain of
+    four) shows.  One chain over each 64-row tile would be 14% (K = 64) or 8% further off; the bound lies
+    halfway, and 0.3% is the spread over draws of this size."""
+    import math
+
+    def predicted(chains):
+        sums, total = [], 0
+        for length in chains:
+            sums += range(8, length + 1, 8)
+            total += length
+            sums += [total] if total > length else []
+        var = 0.0
+        for n in sums:
+            sd = math.sqrt(n / 9)
+            for e in range(-30, 12):
+                inside = math.erf(2.0**(e + 1) / sd / 2**0.5) - math.erf(2.0**e / sd / 2**0.5)
+                var += 2.0**(2 * e - 46) / 12 * inside
+        return math.sqrt(var / (total / 9))
+
+    def measured(K):
+        gen = cuda.Generator(device="cuda").manual_seed(K)
+        A = cuda.empty(64, K, device="cuda").uniform_(-1, 1, generator=gen).half()
+        B = cuda.empty(K, 16384, device="cuda").uniform_(-1, 1, generator=gen).half()
+        T = A.double() @ B.double()
+        return ((mm.gemm(A, B, workspace=False) - T).norm() / T.norm()).item()
+
+    print(f"[gemm 33-64 rows] rounding K {k}", flush=True)
+    steps, tiles = [32] * (k // 32), [min(64, k - i) for i in range(0, k, 64)]
+    bound = (predicted(steps) + predicted(tiles)) / 2 / predicted([32])
+    assert measured(k) / measured(32) <= bound
