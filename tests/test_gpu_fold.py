@@ -336,3 +336,38 @@ def test_gemm_33_to_64_rows_rounding_short(mm, cuda, k):
     steps, tiles = [32] * (k // 32), [min(64, k - i) for i in range(0, k, 64)]
     bound = (predicted(steps) + predicted(tiles)) / 2 / predicted([32])
     assert measured(k) / measured(32) <= bound
+
+
+# (blocks, k_lo, blocks and k_lo of the same K in whole chunks): K up to the line between the kernels (2 x 20,
+# 8 x 9, 4 x 10) and past it, with sums per K step (4 x 18, 6 x 20), per tile (8 x 25) and per fourth one
+@pytest.mark.parametrize("case", [(64, 100, 100, 64), (48, 50, 25, 96), (32, 75, 25, 96), (104, 9, 39, 24), (8, 25, 5, 40),
+                                  (6, 20, 5, 24), (4, 18, 3, 24), (2, 20, 1, 40), (8, 9, 3, 24), (4, 10, 1, 40),
+                                  (400, 5, 25, 80)], ids=lambda c: f"{c[0]}x{c[1]}")
+@pytest.mark.parametrize("form", ["reference", "n_contiguous"])
+def test_fold_padded_k_rounding(mm, cuda, case, form):
+    """Padded K blocks are no further from fp64 than one chain of MFMAs over the same K in whole chunks
+    (0.5%: the spread of a distance over a million outputs)."""
+    def distance(kh, kl):
+        gen = cuda.Generator(device="cuda").manual_seed(kh * kl)
+        a = cuda.empty(2048, kh * kl, device="cuda").uniform_(-1, 1, generator=gen).half()
+        b = cuda.empty(kh * kl, 512, device="cuda").uniform_(-1, 1, generator=gen).half()
+        T = a.double() @ b.double()
+        A = a.reshape(64, 32, kh, kl).permute(0, 2, 1, 3).contiguous()  # [mh][kh][ml][kl]
+        d = mm.ContractDesc()
+        d.m_ext[:], d.n_ext[:], d.k_ext[:] = (64, 32), (1, 512), (kh, kl)
+        d.a_m_stride[:], d.a_k_stride[:] = (kh * 32 * kl, kl), (32 * kl, 1)
+        if form == "reference":  # B [n][kh][kl with 8 elements free after it]
+            B = cuda.zeros(512, kh, kl + 8, dtype=cuda.float16, device="cuda")
+            B[:, :, :kl] = b.t().reshape(512, kh, kl)
+            d.b_k_stride[:], d.b_n_stride[:] = (kl + 8, 1), (0, kh * (kl + 8))
+        else:
+            B = b
+            d.b_k_stride[:], d.b_n_stride[:] = (kl * 512, 512), (0, 1)
+        d.c_m_stride[:], d.c_n_stride[:] = (32 * 512, 512), (0, 1)
+        C = cuda.full((2048, 512), float("nan"), device="cuda")
+        mm.contract(d, A, B, C, workspace=False)
+        return ((C - T).norm() / T.norm()).item()
+
+    kh, kl, kh8, kl8 = case
+    print(f"[fold] rounding {case} {form}", flush=True)
+    assert distance(kh, kl) <= 1.005 * distance(kh8, kl8)
