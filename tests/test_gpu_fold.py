@@ -268,6 +268,12 @@ STREAM64 = [(33, 128, 64, 0), (64, 129, 8, 0), (40, 257, 7, 1), (64, 1000, 1000,
             (57, 16200, 9001, 1), (64, 8192, 16384, 8), (64, 12288, 4096, 0), (35, 17, 100, 2)]
 
 
+# unsplit strips of 64 columns: 256 of them and one more (128-column strips again, 64 ones for K up to 224),
+# last strips of 1, 8 and 63 columns, K past and up to the sums per step, odd K and rows
+STREAM64 += [(64, 16384, 136, 0), (33, 16385, 264, 0), (48, 16392, 224, 8), (61, 16447, 193, 1), (64, 65, 520, 0),
+             (34, 4104, 2049, 7), (39, 127, 225, 0)]
+
+
 @pytest.mark.parametrize("shape", STREAM64, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("ws", [None, False], ids=["workspace", "no_workspace"])
 def test_gemm_33_to_64_rows(mm, cuda, shape, ws):
