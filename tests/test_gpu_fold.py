@@ -117,6 +117,20 @@ def test_fold_padded_k_blocks_n_contiguous(mm, cuda, kl):
         _check(cuda, mm, (2, 130, 1, nl, 3, kl), (A_MID, "kh kl nh nl", "mh ml nh nl"), pads=pads, seed=kl)
 
 
+# the gathering kernel: k runs of 3 one after another in both operands, as given and exchanged (K from 2048);
+# an A strided along K beside a K-major B and a B strided along N beside a K-major A; short padded K
+GATHERED = [((2, 130, 3, 70, 682, 3), (A_MID, "nh nl kh kl")), ((2, 130, 3, 70, 683, 3), (A_MID, "nh nl kh kl")),
+            ((1, 40, 3, 300, 683, 3), (A_MID, "nh nl kh kl")), ((2, 130, 3, 70, 2, 40), ("mh ml kl kh", "nh nl kh kl")),
+            ((2, 130, 2, 70, 3, 40), ("mh kh ml kl", "kh kl nl nh")), ((2, 130, 3, 70, 2, 20), (A_MID, "nh kh nl kl")),
+            ((2, 130, 1, 264, 2, 20), (A_MID, "kh kl nh nl"))]
+
+
+@pytest.mark.parametrize("case", GATHERED, ids=lambda c: "x".join(map(str, c[0])))
+@pytest.mark.parametrize("c_order", ["mh ml nh nl", "nh nl mh ml", "mh nh nl ml"], ids=lambda o: o.replace(" ", ""))
+def test_fold_gathered(mm, cuda, case, c_order):
+    _check(cuda, mm, case[0], (*case[1], c_order))
+
+
 @pytest.mark.parametrize("kl", [40, 64, 100], ids=lambda k: f"kl{k}")
 @pytest.mark.parametrize("offsets", [(1, 0, 0), (0, 3, 1), (7, 5, 0)], ids=str)
 def test_fold_unaligned_operands(mm, cuda, kl, offsets):
