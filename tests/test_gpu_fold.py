@@ -141,6 +141,15 @@ def test_fold_unaligned_operands(mm, cuda, kl, offsets):
            seed=kl)
 
 
+@pytest.mark.parametrize("kl", [96, 128])
+@pytest.mark.parametrize("nl", [300, 1030], ids=["given", "exchanged"])
+def test_fold_wide(mm, cuda, kl, nl):
+    """64-bit addresses (2 GiB from A's first element to its last), K tiles in one block and crossing
+    blocks, edges of the 256x256 tile, the operands as given and exchanged for their m-contiguous C."""
+    _check(cuda, mm, (8, 140, 1, nl, 4, kl), (A_MID, "nh kh nl kl", "mh nh nl ml"), pads=(1 << 18, 0, 0), seed=nl)
+    cuda.cuda.empty_cache()
+
+
 KM = (A_MID, "nh kh nl kl", "mh nh nl ml")
 NM = (A_MID, "kh kl nh nl", "mh ml nh nl")
 # K splits, with and without a workspace: the skinny tiles (1, 16, 32, 33, 64 rows on either side, a
