@@ -33,10 +33,10 @@
  *  - Thread safety: the mutable global state is mmm_gemm_f16f32_noalloc's -- its 64 MiB
  *    device array (shared by every call of that entry point on one GPU) and a mutex-guarded
  *    table of the array's device address per GPU, filled on the first call on each GPU -- and a
- *    mutex-guarded list of the streams on which a call that splits K is being launched.  A
+ *    mutex-guarded list of the workspaces with which a call that splits K is being launched.  A
  *    workspace serves one call at a time: calls on one stream may share one, also from several
  *    host threads (they are ordered, and the two launches of a split call are kept together:
- *    a second thread's split call on that stream waits until both are enqueued); concurrent
+ *    a second thread's split call with that workspace waits until both are enqueued); concurrent
  *    calls on different streams, and graphs that may replay at the same time, need their own.
  */
 #ifndef MMM_H

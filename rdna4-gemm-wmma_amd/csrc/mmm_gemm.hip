@@ -887,7 +887,7 @@ static hipError_t launch_nn(const GemmProblem& p, hipStream_t stream) {
   if (split_tiles < 0 || split_tiles > tiles) return hipErrorInvalidValue;
   const int64_t blocks = tiles - split_tiles + split_tiles * splits;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  const StreamPair pair(pair_stream(splits, stream));
+  const LaunchPair pair(splits > 1 ? p.partials : nullptr);
   // A one-round grid writes all of C after its last K step, with nothing left to overlap, and
   // system-scope write-through stores (sc0 sc1) drain that burst faster.  As half lines they won
   // only where C outgrew the eight XCDs' L2 (32 MB; 256x256 tile: 8192 x 2048 x 2048 +3.1%,
@@ -1182,6 +1182,7 @@ hipError_t launch_gemm_nn(const GemmProblem& p0, int tile_id, hipStream_t stream
                                tiles_n);
           return hipGetLastError();
         }
+        const LaunchPair pair(p.partials);
         if (nt)
           hipLaunchKernelGGL((gemm_nn_persistent_split_kernel<TP, true>), dim3(256), dim3(TP::NT), 0, stream, p, tiles_m,
                              tiles_n);

@@ -74,16 +74,6 @@ bool gemm_nn_persistent(const GemmProblem& p, int tile_id);  // launch as the pe
 // kMaxWorkspaceBytes.
 size_t gemm_nn_workspace_bytes(const GemmProblem& p, int tile_id);
 constexpr size_t kMaxWorkspaceBytes = (size_t)64 << 20;
-// What a StreamPair over the launches of a K split in `splits` ranges holds: an address that stands for
-// the stream (the null stream is one per device; hipStreamPerThread is each thread's own), none if unsplit.
-inline const void* pair_stream(int splits, hipStream_t stream) {
-  if (splits <= 1 || stream == hipStreamPerThread) return nullptr;
-  if ((uintptr_t)stream > 1) return stream;
-  static char null_stream[64];
-  int device = 0;
-  (void)hipGetDevice(&device);
-  return &null_stream[device & 63];
-}
 // A folded problem, with a caller's workspace for a K split's partial tiles (16-byte aligned; null or
 // too small: unsplit) and the bytes that split needs (0: none).
 hipError_t launch_gemm_fold(const FoldProblem& p, void* ws, size_t ws_bytes, hipStream_t stream);

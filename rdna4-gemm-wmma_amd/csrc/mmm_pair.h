@@ -1,11 +1,11 @@
-// Keeps the two launches of a call that splits K together on their stream.
+// Keeps the two launches of a call that splits K together.
 //
-// Such a call writes partial tiles to the caller's workspace in one launch and sums them in the next.
-// Calls on one stream run in order, so they may share a workspace; but with several host threads
-// calling on one stream, another thread's first launch could be enqueued between the two and its
-// partial tiles land before they are summed.  A StreamPair held over both launches admits one thread
-// per stream; threads on other streams are not waited for.  No memory is allocated, and nothing is
-// kept of a call after it.
+// Such a call writes partial tiles to a workspace in one launch and sums them in the next.  Calls on one
+// stream run in order, so they may share a workspace; but with several host threads calling on one
+// stream, another thread's first launch could be enqueued between the two and its partial tiles land
+// before they are summed.  A LaunchPair held over both launches admits one thread per workspace;
+// calls with another workspace are not waited for.  No memory is allocated, and nothing is kept of a
+// call after it.
 #pragma once
 
 #include <condition_variable>
@@ -14,42 +14,51 @@
 
 namespace mmm {
 
-class StreamPair {
+class LaunchPair {
  public:
-  // stream: an address that stands for it (pair_stream in mmm_kernels.h); null: nothing to keep.
-  explicit StreamPair(const void* stream) : stream_(stream) {
-    if (!stream_) return;
+  // workspace: where the partial tiles go; null (unsplit): nothing to keep.
+  explicit LaunchPair(const void* workspace) : workspace_(workspace) {
+    if (!workspace_) return;
     Held& h = held();
     std::unique_lock<std::mutex> lock(h.m);
     int slot;
-    while ((slot = h.slot_for(stream_)) < 0) h.freed.wait(lock);
-    h.streams[slot] = stream_;
+    while ((slot = h.slot_for(workspace_)) < 0) {
+      ++h.waiting;
+      h.freed.wait(lock);
+      --h.waiting;
+    }
+    h.workspaces[slot] = workspace_;
+    if (slot >= h.used) h.used = slot + 1;
   }
-  ~StreamPair() {
-    if (!stream_) return;
+  ~LaunchPair() {
+    if (!workspace_) return;
     Held& h = held();
+    bool wake;
     {
       std::lock_guard<std::mutex> lock(h.m);
-      for (const void*& s : h.streams)
-        if (s == stream_) s = nullptr;
+      for (int i = 0; i < h.used; ++i)
+        if (h.workspaces[i] == workspace_) h.workspaces[i] = nullptr;
+      while (h.used > 0 && !h.workspaces[h.used - 1]) --h.used;
+      wake = h.waiting > 0;
     }
-    h.freed.notify_all();
+    if (wake) h.freed.notify_all();
   }
-  StreamPair(const StreamPair&) = delete;
-  StreamPair& operator=(const StreamPair&) = delete;
+  LaunchPair(const LaunchPair&) = delete;
+  LaunchPair& operator=(const LaunchPair&) = delete;
 
  private:
   static constexpr int kMost = 64;  // threads inside a pair at one moment; one more waits for any of them
   struct Held {
     std::mutex m;
     std::condition_variable freed;
-    const void* streams[kMost] = {};
-    // a free slot if the stream is in none, else -1
-    int slot_for(const void* stream) const {
-      int free = -1;
-      for (int i = kMost - 1; i >= 0; --i) {
-        if (streams[i] == stream) return -1;
-        if (!streams[i]) free = i;
+    int used = 0, waiting = 0;  // slots [used, kMost) are free
+    const void* workspaces[kMost] = {};
+    // a free slot if the workspace is in none, else -1
+    int slot_for(const void* workspace) const {
+      int free = used < kMost ? used : -1;
+      for (int i = used - 1; i >= 0; --i) {
+        if (workspaces[i] == workspace) return -1;
+        if (!workspaces[i]) free = i;
       }
       return free;
     }
@@ -60,7 +69,7 @@ class StreamPair {
     static Held* h = new (mem) Held;
     return *h;
   }
-  const void* stream_;
+  const void* workspace_;
 };
 
 }  // namespace mmm

@@ -672,7 +672,7 @@ static hipError_t launch_wide(const GemmProblem& p, int strips, int splits, floa
                        dim3(strips * splits), dim3(256), 0, stream, p, strips, splits, ws);
   };
   const bool nt = (int64_t)p.K * p.N * 2 >= kNtStreamBytes, shared = p.ldb % 64 != 0;
-  const StreamPair pair(pair_stream(splits, stream));
+  const LaunchPair pair(splits > 1 ? ws : nullptr);
   if (nt && shared)
     launch(std::true_type{}, std::true_type{});
   else if (nt)

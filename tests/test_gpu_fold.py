@@ -209,7 +209,8 @@ def test_fold_splits_threads_one_stream(mm, cuda):
 
 def test_split_entry_points_threads_one_stream(mm, cuda):
     """The C entry points from several host threads on one stream with one workspace, as the header
-    allows: a fold, the streaming kernels' splits and a tile split, each with its own values."""
+    allows: a fold, the streaming kernels' splits, a tile split and a persistent grid's last round, each
+    with its own values."""
     import ctypes as C
     import threading
 
@@ -220,7 +221,7 @@ def test_split_entry_points_threads_one_stream(mm, cuda):
         d, A, B, Cd, T = _check(cuda, mm, (8, 256, 1, 16, 20, 128), KM, seed=s)
         calls.append((L.mmm_contract5d_f16f32_ws, (C.byref(d), ptr(A), ptr(B), ptr(Cd), ptr(ws), ws.numel(), st), Cd, T,
                       (d, A, B)))
-    for M, N, K in ((16, 4096, 4096), (40, 2048, 4096), (256, 256, 8192)):
+    for M, N, K in ((16, 4096, 4096), (40, 2048, 4096), (256, 256, 8192), (4608, 4608, 2048)):
         gen = cuda.Generator(device="cuda").manual_seed(M)
         A, B = (cuda.randint(-4, 5, x, generator=gen, device="cuda").half() for x in ((M, K), (K, N)))
         Cd, T = cuda.empty(M, N, device="cuda"), (A.double() @ B.double()).float()
@@ -231,7 +232,7 @@ def test_split_entry_points_threads_one_stream(mm, cuda):
     wrong = []
 
     def work(i, fn, args, Cd, T, keep):
-        rc = [fn(*args) for _ in range(200)]
+        rc = [fn(*args) for _ in range(100)]
         cuda.cuda.synchronize()
         if any(rc) or not cuda.equal(Cd, T):
             wrong.append(i)

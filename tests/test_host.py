@@ -491,9 +491,9 @@ def test_captured_calls_get_their_own_workspace(mm, monkeypatch):
     assert mm._ws_args(None, dev, st, lambda: 4096) == (None, None, 0)
 
 
-def test_stream_pair_holds_one_thread_per_stream(tmp_path):
-    """csrc/mmm_pair.h, under which a split call's two launches are enqueued: threads on one stream never
-    interleave, a thread on another stream does not wait, and more threads than slots all get through."""
+def test_launch_pair_holds_one_thread_per_workspace(tmp_path):
+    """csrc/mmm_pair.h, under which a split call's two launches are enqueued: threads with one workspace
+    never interleave, a thread with another does not wait, and more threads than slots all get through."""
     src = tmp_path / "pair.cpp"
     src.write_text("""
 #include <atomic>
@@ -503,14 +503,14 @@ def test_stream_pair_holds_one_thread_per_stream(tmp_path):
 #include <vector>
 #include "mmm_pair.h"
 int main() {
-  static char streams[200];
+  static char ws[200];
   std::atomic<int> inside[200] = {}, mixed{0}, done{0};
   std::vector<std::thread> threads;
   for (int t = 0; t < 16; ++t)
     threads.emplace_back([&, t] {
       for (int i = 0; i < 2000; ++i) {
         const int s = (t + i) % 3;
-        mmm::StreamPair pair(&streams[s]);
+        mmm::LaunchPair pair(&ws[s]);
         if (inside[s].fetch_add(1) != 0) ++mixed;
         if (i % 64 == 0) std::this_thread::yield();
         inside[s].fetch_sub(1);
@@ -519,19 +519,19 @@ int main() {
   for (auto& t : threads) t.join();
   if (mixed) return 1;
   {
-    mmm::StreamPair a(&streams[0]), unsplit(nullptr), unsplit2(nullptr);
-    auto other = std::async(std::launch::async, [&] { mmm::StreamPair b(&streams[1]); });
+    mmm::LaunchPair a(&ws[0]), unsplit(nullptr), unsplit2(nullptr);
+    auto other = std::async(std::launch::async, [&] { mmm::LaunchPair b(&ws[1]); });
     if (other.wait_for(std::chrono::seconds(20)) != std::future_status::ready) return 2;
-    auto same = std::async(std::launch::async, [&] { mmm::StreamPair b(&streams[0]); ++done; });
+    auto same = std::async(std::launch::async, [&] { mmm::LaunchPair b(&ws[0]); ++done; });
     if (same.wait_for(std::chrono::milliseconds(100)) == std::future_status::ready) return 3;
-    a.~StreamPair();
+    a.~LaunchPair();
     same.wait();
-    new (&a) mmm::StreamPair(nullptr);
+    new (&a) mmm::LaunchPair(nullptr);
   }
   std::vector<std::thread> many;
   for (int t = 0; t < 200; ++t)
     many.emplace_back([&, t] {
-      mmm::StreamPair pair(&streams[t]);
+      mmm::LaunchPair pair(&ws[t]);
       std::this_thread::sleep_for(std::chrono::milliseconds(2));
       ++done;
     });
@@ -545,12 +545,14 @@ int main() {
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
     assert subprocess.run([str(exe)], timeout=60).returncode == 0
-    # every pair of launches in the library is under one
-    for name, launches in (("mmm_gemm.hip", "reduce_tiles_kernel<"), ("mmm_skinny.hip", "reduce_splits_kernel<"),
-                           ("mmm_fold.hip", "reduce_fold_kernel<")):
-        text = open(os.path.join(csrc, name)).read()
-        at = text.index("hipLaunchKernelGGL((" + launches)
-        assert "StreamPair pair(" in text[text.rindex("static hipError_t ", 0, at):at], name
+    # every reduction in the library is launched under one, taken after the function or case it is in began
+    for name, kernel, n in (("mmm_gemm.hip", "reduce_tiles_kernel<", 2), ("mmm_skinny.hip", "reduce_splits_kernel<", 1),
+                            ("mmm_fold.hip", "reduce_fold_kernel<", 1)):
+        parts = open(os.path.join(csrc, name)).read().split("hipLaunchKernelGGL((" + kernel)
+        assert len(parts) == n + 1, name
+        for before in parts[:-1]:
+            start = max(before.rfind("hipError_t launch_"), before.rfind("      case "))
+            assert "const LaunchPair pair(" in before[start:], name
 
 
 def test_launches_do_not_wait_for_each_other(mm, monkeypatch):
