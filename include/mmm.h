@@ -158,10 +158,12 @@ typedef struct mmm_gemm_plan {
                                               interior tiles over several rounds) */
     int64_t workspace_bytes;               /* workspace the splits need (mmm_gemm_f16f32_ws);
                                               the split counts above assume it is given, and so
-                                              does the kernel choice for M <= 64: without a
-                                              workspace, aligned problems whose 128-column strips
-                                              fill rounds of 256 workgroups less than 1/1.8 run
-                                              on the streaming kernel, not on tiles */
+                                              does the kernel choice: without a workspace,
+                                              problems of M <= 64 and aligned rows whose 128-column
+                                              strips fill rounds of 256 workgroups less than 1/1.8
+                                              run on the streaming kernel, not on tiles, and grids
+                                              of a few 128x128 tiles past whole rounds stay on
+                                              those tiles */
     int stream_columns;                    /* columns of C per streaming workgroup: 32 (K split
                                               among one workgroup's waves), 128, or 256 (long
                                               K streams); 0: no streaming kernel.  33 to 64 rows

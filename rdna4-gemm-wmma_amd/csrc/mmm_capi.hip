@@ -136,7 +136,7 @@ constexpr double kPartialRoundBoost = 0.3;
 // the smaller tiles' rate is operand loads per flop ((BM + BN) / (BM * BN): 1.5x for the narrow
 // tiles, 2x for 128x128, 4x for 64x64), which saturate the address unit (TA busy 0.48 for
 // 256x256, 0.59-0.65 narrow, 0.83 for 128x128, 0.89 for 64x64); no tile has LDS bank conflicts.
-// The narrow tiles are priced at 0.82 (128x128: below); 192x192 and 64x64 at 0.86 and 0.30,
+// The narrow tiles are priced at 0.82 and 128x128 at 0.76; 192x192 and 64x64 at 0.86 and 0.30,
 // the values that pick the faster tile on the shapes
 // measured for them: 192x192 on 3072^3, 3072^2 x 8192, 4357 x 4095 x 4111 and the 4-way K split
 // of 1536^2 x 12288 (937 TFLOP/s against 864 for a 7-way split of 256x256 tiles), 256x256 on
@@ -158,34 +158,31 @@ constexpr double kEff64 = 0.30, kEffNarrow = 0.82, kEff192 = 0.86;
 // Reduction traffic of a K split as tile_cost prices it against other tiles (the split decision
 // itself, gemm_nn_split, uses kSplitTrafficBps).
 constexpr double kSplitCostBps = 5e12;
-// The 128x128 tile's 0.76 is its rate in multi-round grids. Shorter ones it runs slower than that
-// against the wider tiles, as timed with every tile forced on 466 shapes (operands rotating through
-// HBM, 65 to 8192 rows, 64 to 28672 columns, K 64 to 28672). On 288 further shapes, not used
-// for the prices, 23 picks changed, all for the faster, and the pick went from 3.8% to 2.6% behind the
-// fastest tile on average:
-//  * One round, unsplit (DeepTile128): 0.66, 448 x 4168 x 3776 38.7 -> 31.1 us on 256x128, 1376 x 2488 x
-//    9485 118.3 -> 96.5 on 256x256. At 0.64 448 x 8192 x 8192, 256 tiles, leaves it and loses 5%.
-//  * A K split of the whole grid: 0.64, 1400 x 1024 x 6488 43.6 -> 33.9 us on 128x256, 384 x 4096 x
-//    4096 30.1 -> 26.9.
-//  * Neither at 160 rows or columns or fewer, where wider tiles are half empty: 0.70 and 0.76 (with
-//    the prices above 136 x 4096 x 11008 34.7 -> 38.3 us, 72 x 28672 x 8192 93.8 -> 100.0).
-//  * Up to 64 tiles past whole rounds, run as K ranges: 0.60. Two workgroups share a CU there, and the
-//    ranges slow the whole tiles beside them: 4160 x 1024 x 8192 (8 tiles past 256) 110.9 -> 82.7 us on
-//    256x256, 288 x 11298 x 6696 99.7 -> 80.1 on 192x192, 576 x 8192 x 28672 392 -> 330. Not
-//    with K below 4096 or more tiles left, where it is the faster one: 1720 x 2352 x 2976 47.2
-//    against 55.0 on 256x128, 3456 x 1600 x 7856 (95 tiles) 120.4 against 137.3.
-static double eff128(const GemmProblem& p, const TileSplit& sp, double tiles) {
-  const bool narrow = std::min(p.M, p.N) <= 160;
-  if (sp.splits > 1 && sp.tiles < tiles) return p.K >= 4096 && sp.tiles <= 64 ? 0.60 : 0.76;
-  if (sp.splits > 1) return narrow ? 0.76 : 0.64;
-  return tiles > 256.0 ? 0.76 : narrow ? 0.70 : 0.66;
-}
-static double tile_cost(const GemmProblem& p, int tile, int* splits_out) {
-  static const double eff_of[kTileCount] = {1.0, kEffNarrow, kEffNarrow, 0.0, kEff64, kEff192};
+// The 128x128 tile: 0.76 in multi-round grids and K splits; in an unsplit launch of one round, where it
+// runs its 3-stage ring (DeepTile128), 0.70: that still picks it at 512 x 8192 x 8192 (867-919 TFLOP/s
+// against 842-876 for a 4-way K split of 64 256x256 tiles) and gives 448-512 x 4096 x 4096 to 256x128
+// tiles (measured with B rotating through HBM 521 against 399 TFLOP/s at 512 rows, B resident +8%).
+// Priced lower (0.60 to 0.66) in those forms, it gave way on 160 of 4418 shapes (65 to 8192 rows,
+// 64 to 16384 columns and K): 9% faster on average, but 22 slower by 3 to 24% (3384 x 776 x 7840
+// 60.8 -> 75.3 us on 256x128, 6730 x 178 x 5522 35.6 -> 40.7 on 192x192) and 49 further from fp64, by up to
+// 2.1x, on tiles that split K less (793 x 1151 x 3393 unsplit on 64x64).
+constexpr double kEff128 = 0.76, kEff128Deep = 0.70;
+// One form of launch is priced lower: whole rounds and up to 64 tiles more, run as K ranges. Two
+// workgroups share a CU there, and the ranges slow the whole tiles beside them: 2752 x 1600 x 10560 (25
+// tiles past 256) at 0.70 of its time on 256x256, 4274 x 930 x 8708 0.66 on 192x192, 384 x 11072 x 5376 0.68. Not
+// with K below 4096 or more tiles left, where it is the faster one: 1720 x 2352 x 2976 47.2
+// against 55.0 on 256x128, 3456 x 1600 x 7856 (95 tiles) 120.4 against 137.3. And not for an unsplit tile
+// (7400 x 608 x 8976 152.6 -> 171.5 us on 256x128, and 5% further from fp64), nor without a workspace
+// (pick_tile): the larger tiles then leave most of the chip idle, 2752 x 1600 x 10560 146 -> 225 us.
+constexpr double kEff128Tail = 0.60;
+static double tile_cost(const GemmProblem& p, int tile, int* splits_out, bool price_tail = false) {
+  static const double eff_of[kTileCount] = {1.0, kEffNarrow, kEffNarrow, kEff128, kEff64, kEff192};
   const int bm = tile_bm(tile), bn = tile_bn(tile);
   const TileSplit sp = gemm_nn_split(p, tile);
   const double tiles = (double)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
-  const double tile_eff = tile == kTile128x128 ? eff128(p, sp, tiles) : eff_of[tile];
+  double tile_eff = eff_of[tile];
+  if (tile == kTile128x128 && sp.splits <= 1 && tiles <= 256.0) tile_eff = kEff128Deep;
+  if (tile == kTile128x128 && price_tail) tile_eff = kEff128Tail;
   const double per_cu_flops = 4.8e12;  // sustained MFMA rate of one CU under load (256x256 at 8192^3)
   // A round with `active` of its 256 slots busy runs each CU faster: the chip is then below its
   // power cap and keeps a higher clock.  Fitted with the prices above (3072^3 ran 878 TFLOP/s
@@ -221,19 +218,29 @@ static double tile_cost(const GemmProblem& p, int tile, int* splits_out) {
 // The cheapest tile by tile_cost; a smaller tile must win by 3% (where the estimates are that
 // close, the measured times are too, and the larger tile reads less LDS per MAC).
 static int pick_tile(const GemmProblem& p) {
-  int best = kTile256x256, s = 1;
-  double best_cost = 1e300;
-  for (int tile : {kTile256x256, kTile256x128, kTile128x256, kTile128x128, kTile64x64, kTile192x192}) {
-    if (tile == kTile192x192 && !gemm_nn_direct_to_lds(p, tile)) continue;  // direct-to-LDS only
-    const double c = tile_cost(p, tile, &s);
-    if (c < best_cost * 0.97) {
-      best_cost = c;
-      best = tile;
+  auto cheapest = [&](bool price_tail, int* splits) {
+    int best = kTile256x256, s = 1;
+    double best_cost = 1e300;
+    for (int tile : {kTile256x256, kTile256x128, kTile128x256, kTile128x128, kTile64x64, kTile192x192}) {
+      if (tile == kTile192x192 && !gemm_nn_direct_to_lds(p, tile)) continue;  // direct-to-LDS only
+      const double c = tile_cost(p, tile, &s, price_tail);
+      if (c < best_cost * 0.97) {
+        best_cost = c;
+        best = tile;
+        *splits = s;
+      }
     }
-  }
-  return best;
+    return best;
+  };
+  int splits = 1;
+  const int best = cheapest(false, &splits);
+  if (best != kTile128x128 || splits < 2 || p.K < 4096 || p.ws_absent) return best;
+  const int last = gemm_nn_split(p, best).tiles;
+  const int64_t tiles = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128);
+  if (last == tiles || last > 64) return best;
+  const int other = cheapest(true, &splits);  // kEff128Tail
+  return splits > 1 ? other : best;
 }
-
 
 // What mmm_gemm_f16f32 launches for a validated problem.
 struct GemmPlan {

@@ -575,3 +575,17 @@ def test_launches_do_not_wait_for_each_other(mm, monkeypatch):
     one.join(60)
     two.join(60)
     assert passed
+
+
+def test_gemm_plan_128_tile_forms(mm):
+    """The 128x128 tile gives way where a few of its tiles past whole rounds would run as K ranges beside
+    them, to a split larger tile only; its one-round and whole-grid K splits stay (each pick measured)."""
+    def plan(*s):
+        p = mm.gemm_plan(*s)
+        return p["block_m"], p["block_n"], p["tile_splits"]
+
+    assert plan(2752, 1600, 10560) == (256, 256, 3) and plan(4274, 930, 8708) == (192, 192, 2)
+    assert plan(1720, 2352, 2976)[:2] == (128, 128)  # K below 4096
+    assert plan(7400, 608, 8976) == (128, 128, 7)    # 256x128 would run unsplit
+    for s in ((3384, 776, 7840), (6730, 178, 5522), (793, 1151, 3393), (688, 808, 2696)):
+        assert plan(*s)[:2] == (128, 128), s
