@@ -78,9 +78,9 @@ __global__ __launch_bounds__(T::NT, nn_launch_occupancy<T>()) void gemm_nn_kerne
   const bool split_block = (int)blockIdx.x >= whole;
   const int nsplit = split_block ? ksplit : 1;
   int q = 0, j = -1, tm, tn;
-  if (split_block) split_item((int)blockIdx.x, whole, p.split_tiles, ksplit, &q, &j);
+  if (split_block) split_item((int)blockIdx.x, whole, p.split_tiles, ksplit, p.split_major, &q, &j);
   q = __builtin_amdgcn_readfirstlane(q);
-  tile_of_item((int)blockIdx.x, j, whole, ksplit, tiles_m, tiles_n, &tm, &tn);
+  tile_of_item((int)blockIdx.x, j, whole, p.split_major, tiles_m, tiles_n, &tm, &tn);
   // The tile origin is uniform; readfirstlane keeps it (and everything derived from it, such
   // as the buffer descriptors) in SGPRs -- the integer divisions above are expanded on the VALU.
   const int m0 = __builtin_amdgcn_readfirstlane(tm * T::BM), n0 = __builtin_amdgcn_readfirstlane(tn * T::BN);
@@ -860,7 +860,7 @@ __global__ __launch_bounds__(256) void reduce_tiles_kernel(GemmProblem p, int ti
   const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int j = (int)(g / F4), e = (int)(g % F4);
   int tm, tn;
-  tile_of_item(0, j, first, splits, tiles_m, tiles_n, &tm, &tn);
+  tile_of_item(0, j, first, p.split_major, tiles_m, tiles_n, &tm, &tn);
   const int r = e / (BN / 4), c = 4 * (e % (BN / 4));
   const int m = tm * BM + r, n = tn * BN + c;
   if (m >= p.M || n >= p.N) return;
@@ -878,7 +878,8 @@ __global__ __launch_bounds__(256) void reduce_tiles_kernel(GemmProblem p, int ti
 
 
 template <class T, bool GENERIC>
-static hipError_t launch_nn(const GemmProblem& p, hipStream_t stream) {
+static hipError_t launch_nn(const GemmProblem& p0, hipStream_t stream) {
+  GemmProblem p = p0;
   const int tiles_m = (p.M + T::BM - 1) / T::BM;
   const int tiles_n = (p.N + T::BN - 1) / T::BN;
   const int64_t tiles = (int64_t)tiles_m * tiles_n;
@@ -887,6 +888,8 @@ static hipError_t launch_nn(const GemmProblem& p, hipStream_t stream) {
   if (split_tiles < 0 || split_tiles > tiles) return hipErrorInvalidValue;
   const int64_t blocks = tiles - split_tiles + split_tiles * splits;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+  p.split_major = splits > 1 && split_major((int)(tiles - split_tiles), splits, T::BM, T::BN,
+                                            (p.K + 63) / 64 / splits, ((int64_t)p.M + p.N) * p.K * 2);
   const LaunchPair pair(splits > 1 ? p.partials : nullptr);
   // A one-round grid writes all of C after its last K step, with nothing left to overlap, and
   // system-scope write-through stores (sc0 sc1) drain that burst faster.  As half lines they won

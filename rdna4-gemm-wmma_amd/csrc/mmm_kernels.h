@@ -21,6 +21,7 @@ struct GemmProblem {
                    // of 8, or rows not 16-byte aligned): patched chunks or a VGPR gather
   int k_splits;    // tile kernel: K ranges computed by separate workgroups (<= 1: none)
   int split_tiles; // k_splits > 1: the last split_tiles tiles in dispatch order are split
+  bool split_major; // k_splits > 1: order of a grid whose every tile is split (mmm_tile_map.h)
   float* partials; // k_splits > 1: [split tile][split][BM][BN] fp32 partial tiles
   float* ws;       // caller's workspace for K splits (16-byte aligned), or null: no split
   size_t ws_bytes; // its size

@@ -14,6 +14,8 @@
 //     that shares 4 A panels and 8 B panels in that XCD's L2.
 #pragma once
 
+#include <stdint.h>
+
 #ifdef __HIPCC__
 #define MMM_HD __host__ __device__ __forceinline__
 #else
@@ -46,23 +48,29 @@ MMM_HD void tile_of_block(int b, int tiles_m, int tiles_n, int group_m, int* tm,
 
 // A grid in which the tiles from `whole` on run as `splits` K ranges (whole == 0: every tile).  Block b
 // of those is K range q of split tile j, block whole + q * split_tiles + j; with every tile split into
-// more than two ranges, the blocks are numbered so that each XCD takes a contiguous run of the items
-// (q, j): it then reads as few K ranges as possible, and a slice of A or B is fetched by one or two L2s
-// instead of by every one that holds a tile.  Measured on MI355X (B from HBM): 64 x 4096 x 16384 34.5
-// -> 30.1 us, 128 x 4096 x 4096 20.1 -> 18.2, 2000 x 1000 x 8192 48.6 -> 45.4, 1536^2 x 12288 63.4 ->
-// 61.4; with two ranges 128 x 14336 x 4096 38.3 -> 39.3.
-MMM_HD bool split_major(int whole, int splits) { return whole == 0 && splits > 2; }
+// more than two ranges (`major`, split_major), the blocks are numbered so that each XCD takes a contiguous
+// run of the items (q, j): it then reads as few K ranges as possible, and a slice of A or B is fetched by one
+// or two L2s instead of by every one that holds a tile.  Measured on MI355X (B from HBM): 64 x 4096 x 16384
+// 34.5 -> 30.1 us, 128 x 4096 x 4096 20.1 -> 18.2, 2000 x 1000 x 8192 48.6 -> 45.4, 1536^2 x 12288 63.4 ->
+// 61.4; with two ranges 128 x 14336 x 4096 38.3 -> 39.3.  Not on 128x128 tiles over ranges of fewer than 16 K
+// tiles of operands of 8 to 20 MB, which the L2s hold either way: there 704 x 1024 x 2816 took 17.3 us
+// against 13.9, 448 x 2368 x 2816 17.7 against 15.7, and 64 shapes of that kind 2.6% more on average (one,
+// three or eight sets of buffers in turn made no difference); smaller operands 2% less, larger ones 7 to 10%.
+MMM_HD bool split_major(int whole, int splits, int bm, int bn, int range_k_tiles, int64_t operand_bytes) {
+  if (whole != 0 || splits <= 2) return false;
+  return !(bm == 128 && bn == 128 && range_k_tiles < 16 && operand_bytes >= 8000000 && operand_bytes < 20000000);
+}
 
-MMM_HD void split_item(int b, int whole, int split_tiles, int splits, int* q, int* j) {
-  const int v = split_major(whole, splits) ? xcd_compact(b, split_tiles * splits) : b - whole;
+MMM_HD void split_item(int b, int whole, int split_tiles, int splits, bool major, int* q, int* j) {
+  const int v = major ? xcd_compact(b, split_tiles * splits) : b - whole;
   *q = v / split_tiles;
   *j = v - *q * split_tiles;
 }
 
 // The tile of block b (unsplit; j < 0) or of split tile j.
-MMM_HD void tile_of_item(int b, int j, int whole, int splits, int tiles_m, int tiles_n, int* tm, int* tn) {
+MMM_HD void tile_of_item(int b, int j, int whole, bool major, int tiles_m, int tiles_n, int* tm, int* tn) {
   int v = j < 0 ? b : whole + j;
-  if (j < 0 || !split_major(whole, splits)) v = xcd_compact(v, tiles_m * tiles_n);
+  if (j < 0 || !major) v = xcd_compact(v, tiles_m * tiles_n);
   grouped_tile(v, tiles_m, tiles_n, 4, tm, tn);
 }
 
