@@ -166,9 +166,9 @@ typedef struct mmm_gemm_plan {
                                               those tiles */
     int stream_columns;                    /* columns of C per streaming workgroup: 32 (K split
                                               among one workgroup's waves), 128, or 256 (long
-                                              K streams); 0: no streaming kernel.  33 to 64 rows
-                                              unsplit: a strip of 128 may run as two workgroups
-                                              of 64 columns (stream_workgroups counts those) */
+                                              K streams); 0: no streaming kernel.  33 to 64 rows:
+                                              a strip of 128 may run as two workgroups of 64
+                                              columns (stream_workgroups counts those) */
 } mmm_gemm_plan;
 
 /*

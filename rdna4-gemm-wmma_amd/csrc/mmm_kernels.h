@@ -80,7 +80,7 @@ constexpr size_t kMaxWorkspaceBytes = (size_t)64 << 20;
 hipError_t launch_gemm_fold(const FoldProblem& p, void* ws, size_t ws_bytes, hipStream_t stream);
 size_t gemm_fold_workspace_bytes(const FoldProblem& p);
 // Row-major GEMMs of 33 to 64 rows on the fold kernel's skinny tiles: strips of 128 or 256 columns x
-// `splits` K ranges (> 1: partial tiles of 64 rows in `partials`), or unsplit strips of 64 columns, which K
+// `splits` K ranges (> 1: partial tiles of 64 rows in `partials`), or of 64 columns, which K
 // of up to kStepSumsMost steps of 32 always takes.  ok: operands it can address.
 constexpr int kStepSumsMost = 7;
 bool gemm_stream64_ok(const GemmProblem& p);

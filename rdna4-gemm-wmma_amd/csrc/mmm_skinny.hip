@@ -589,10 +589,12 @@ static StreamShape stream_shape(const GemmProblem& p) {
   return {mr, 128, strips, splits};
 }
 
-// 33 to 64 rows in one K range a strip: workgroups of 64 columns, two a strip, while they fit one round of
-// the chip (GemmTile64x64 has both sides), and with K of up to kStepSumsMost steps of 32 always.
-static bool half_strips(const GemmProblem& p, int splits) {
-  return stream_mr(p.M) == 4 && splits == 1 && ((p.N + 63) / 64 <= 256 || p.K <= 32 * kStepSumsMost);
+// 33 to 64 rows on 128-column strips: workgroups of 64 columns, two a strip, while they and their K ranges
+// fit one round of the chip (GemmTile64x64 has both sides), and with K of up to kStepSumsMost steps of 32
+// always.  The partial tiles take no more of the workspace than whole strips' do.
+static bool half_strips(const GemmProblem& p, int columns, int splits) {
+  if (stream_mr(p.M) != 4 || columns != 128) return false;
+  return (p.N + 63) / 64 * splits <= 256 || p.K <= 32 * kStepSumsMost;
 }
 
 int skinny_splits(const GemmProblem& p) { return stream_shape(p).splits; }
@@ -641,7 +643,7 @@ size_t skinny_workspace_bytes(const GemmProblem& p) {
 
 int skinny_workgroups(const GemmProblem& p) {
   const StreamShape sh = stream_shape(p);
-  if (half_strips(p, sh.splits)) return (p.N + 63) / 64;
+  if (half_strips(p, sh.ns, sh.splits)) return (p.N + 63) / 64 * sh.splits;
   return sh.splits ? sh.strips * sh.splits : (p.N + kNS - 1) / kNS;
 }
 
@@ -706,7 +708,7 @@ hipError_t launch_gemm_skinny(const GemmProblem& p0, hipStream_t stream) {
         return sh.ns == 256 ? launch_wide<2, 256>(p, sh.strips, sh.splits, ws, stream)
                             : launch_wide<2, 128>(p, sh.strips, sh.splits, ws, stream);
       default:
-        return launch_gemm_stream64(p, half_strips(p, sh.splits) ? 64 : sh.ns, sh.splits, ws, stream);
+        return launch_gemm_stream64(p, half_strips(p, sh.ns, sh.splits) ? 64 : sh.ns, sh.splits, ws, stream);
     }
   }
   // wave-split kernel (M <= 16): no caller workspace
