@@ -82,7 +82,7 @@ size_t gemm_fold_workspace_bytes(const FoldProblem& p);
 // Row-major GEMMs of 33 to 64 rows on the fold kernel's skinny tiles: strips of 128 or 256 columns x
 // `splits` K ranges (> 1: partial tiles of 64 rows in `partials`), or of 64 columns, which K
 // of up to kStepSumsMost steps of 32 always takes.  ok: operands it can address.
-constexpr int kStepSumsMost = 7;
+constexpr int kStepSumsMost = 10;
 bool gemm_stream64_ok(const GemmProblem& p);
 hipError_t launch_gemm_stream64(const GemmProblem& p, int columns, int splits, float* partials, hipStream_t stream);
 // The operand-path probe (lds_mfma_probe_kernel): M, N multiples of 256, K of 128, row-major A
