@@ -19,7 +19,6 @@ namespace mmm {
 // Fragment offsets a wave keeps per K-step (A) or per B fragment: at most kMaxOff of each.
 constexpr int kMaxOff = 8;
 
-
 // Block tile BM x BN, K step BK (32 or 64), WGM x WGN waves, STAGES-deep LDS ring, OCC
 // workgroups per CU targeted by the launch bounds (OCC > 1 caps registers accordingly), MFMA
 // shape MF: 32 = v_mfma_f32_32x32x16_f16, 16 = v_mfma_f32_16x16x32_f16 (same MACs per LDS byte;
@@ -592,8 +591,6 @@ using DmaTile = typename DmaCfg<BM, BN>::T;
 // than 3; then eight waves of 16x16x32 instead of four of 32x32x16: 2048^3 601 -> 645, 2048^2 x
 // 4096 760 -> 822, 1024^2 x 8192 538 -> 564, 512 x 8192 x 8192 783 -> 852.
 using DeepTile128 = Tile<128, 128, 2, 4, 64, 3, 1, 16>;
-// The folded direct-to-LDS kernel: the 256x256 tile's waves and ring.
-using FoldDmaTile = Tile256;
 // Register-staged path: 64-deep stages, double-buffered.
 template <int BM, int BN>
 using RegTile = Tile<BM, BN, 2, 2, 64, 2>;
