@@ -152,10 +152,10 @@ def test_fold_wide(mm, cuda, kl, nl):
 
 KM = (A_MID, "nh kh nl kl", "mh nh nl ml")
 NM = (A_MID, "kh kl nh nl", "mh ml nh nl")
-# K splits, with and without a workspace: the skinny tiles (1, 16, 32, 33, 64 rows on either side, a
-# side of 65 on square tiles), ends of N inside a tile, K blocks per tile, per lane and padded, a split
-# of a partly filled last round (272 tiles of 256 x 256), and streams of 64 MiB and more against 16, 33, 17, 64, 30 and 24 rows
-# (the last six; NT loads from 96 MiB)
+# K splits, with and without a workspace, on the square tiles: 1, 16, 32, 33, 64 and 65 rows on either side, ends
+# of N inside a tile, K blocks per tile, per lane and padded, a split of a partly filled last round (272 tiles
+# of 256 x 256); and on the skinny tiles, streams of 64 MiB and more (K tiles inside one block) against 16, 33,
+# 17, 64, 30 and 24 rows (the last six; NT loads from 96 MiB)
 SPLITS = [((1, 1, 4, 300, 20, 128), KM), ((4, 300, 1, 16, 20, 128), KM), ((4, 301, 1, 32, 33, 72), KM),
           ((3, 11, 4, 300, 20, 100), KM), ((2, 32, 4, 1024, 24, 100), KM), ((5, 13, 4, 300, 20, 128), KM),
           ((1, 16, 1, 1027, 20, 128), NM), ((2, 32, 1, 2045, 31, 72), NM), ((2, 8, 4, 64, 31, 50), (A_MID, "kh nh kl nl",
@@ -286,16 +286,20 @@ def test_fold_split_graphs_at_once(mm, cuda, bound, monkeypatch):
 
 
 # 33 to 64 rows of a row-major GEMM on the fold kernel's skinny tiles: one K tile and K ends inside one,
-# odd K and N, a last strip of one column, rows at 2-byte alignment, 256-column strips, one strip, B from
-# 96 MiB (non-temporal); the view's padding is NaN
+# odd K and N, a last strip of one column, rows at 2-byte alignment, 256-column strips (odd N, K ending inside a
+# chunk and between chunks), one strip, B from 96 MiB (non-temporal); the view's padding is NaN
 STREAM64 = [(33, 128, 64, 0), (64, 129, 8, 0), (40, 257, 7, 1), (64, 1000, 1000, 8), (50, 2041, 1031, 3), (33, 16, 9000, 0),
             (57, 16200, 9001, 1), (64, 8192, 16384, 8), (64, 12288, 4096, 0), (35, 17, 100, 2)]
+STREAM64 += [(57, 16200, 9001, 8), (57, 16201, 9008, 7), (33, 16398, 8197, 2), (64, 12288, 4160, 0), (64, 20000, 4096, 0)]
 
 
 # unsplit strips of 64 columns: 256 of them and one more (128-column strips again, 64 ones for K up to 224),
 # last strips of 1, 8 and 63 columns, K past and up to the sums per step, odd K and rows
-STREAM64 += [(64, 16384, 136, 0), (33, 16385, 264, 0), (48, 16392, 224, 8), (61, 16447, 193, 1), (64, 65, 520, 0),
+STREAM64 += [(64, 16384, 136, 0), (33, 16385, 264, 0), (48, 16392, 224, 8), (61, 16447, 193, 1), (64, 65, 1100, 0),
              (34, 4104, 2049, 7), (39, 127, 225, 0)]
+
+
+COLUMNS_256 = [(57, 16200, 9001, 8), (64, 8192, 16384, 8), (57, 16201, 9008, 7), (33, 16398, 8197, 2)]
 
 
 @pytest.mark.parametrize("shape", STREAM64, ids=lambda s: "x".join(map(str, s)))
@@ -312,6 +316,11 @@ def test_gemm_33_to_64_rows(mm, cuda, shape, ws):
     A, B = view(M, K), view(K, N)
     C = cuda.full((M, N), float("nan"), dtype=cuda.float32, device="cuda")
     print(f"[gemm 33-64 rows] {shape} workspace {ws is None}", flush=True)
+    plan = mm.gemm_plan(M, N, K, lda=K + pad, ldb=N + pad)
+    if shape == (64, 12288, 4096, 0):  # with a workspace this one runs on 64x64 tiles: streamed without only
+        assert plan["kernel"] == "tile"
+    else:
+        assert plan["kernel"] == "stream" and plan["stream_columns"] == (256 if shape in COLUMNS_256 else 128)
     mm.gemm(A, B, C, workspace=ws)
     T = (A.double() @ B.double()).float()
     assert cuda.equal(C, T), f"{int((C != T).sum().item())} outputs differ"
