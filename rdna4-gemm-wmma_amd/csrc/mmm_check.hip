@@ -19,7 +19,7 @@
 // accumulator's type, so the loop is LDS reads and FMAs only.  K stages are double-buffered through
 // registers, deeper with fewer outputs per thread (a stage has to cover the next one's loads: 64 x 64
 // x 2048 119 us with 16 k a stage, 98 with 64).  Measured on MI355X, T and S, against the kernel before
-// (4x4 outputs, converted per use, multiply, add and |.| apart): 2048^3 1947 -> 682 us (50 TFLOP/s),
+// (4x4 outputs, converted per use, multiply, add and |.| apart): 2048^3 1939 -> 660 us (52 TFLOP/s),
 // 4096 x 4096 x 1024 3559 -> 1231, 1000^3 366 -> 142, 512 x 512 x 2048 647 -> 106, 64 x 64 x 2048 642 ->
 // 98; T alone 2048^3 1931 -> 458, the fp32 mode 562 -> 307.  Few outputs are bound by one k after the
 // other per output, which the defined order asks for.

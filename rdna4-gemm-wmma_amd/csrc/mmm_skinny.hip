@@ -575,12 +575,13 @@ static StreamShape stream_shape(const GemmProblem& p) {
   // 17 to 32 rows: 32 x 12288 x 16384 (819 rows per wave) +8.8%, 17 x 16384 x 16384 (1024)
   // +5.2%, 32 x 8192 x 28672 (896) +3.8%, 24 x 8192 x 16384 (512) +2.3%, 32 x 16384 x 8192 (512)
   // +0.9%; 32 x 8192 x 12288 (384) +-0, 32 x 6144 x 16384 (410) -2.2%, 32 x 8192 x 8192 (256)
-  // -1.3%, 32 x 4096 x 8192 (128) -11%.  33 to 64 rows: 48 x 12288 x 16384 (819) +19.5% (240
-  // workgroups instead of 192), 64 x 8192 x 28672 (896) +4.2%, 64 x 8192 x 16384 (512) +1.9%,
-  // 40 x 16384 x 16384 (1024) +1.2%, 64 x 16384 x 8192 (512) +1.0%; 48 x 8192 x 12288 (384)
-  // -2.5%, 64 x 4096 x 14336 (224) -1.0%, 64 x 8192 x 8192 (256) -0.4%.  From an unsplit
-  // 128-column grid only 33 to 64 rows, whose 128-column slots are one third A: 64 x 28672 x 8192
-  // +6.6% (1024 rows per wave), 48 x 28672 x 8192 +2.7% (16 rows: -1.0%, above).
+  // -1.3%, 32 x 4096 x 8192 (128) -11%.  33 to 64 rows, on the tiles that the waves share (us, 128 against
+  // 256 columns): 48 x 12288 x 16384 80.5 against 70.7, 64 x 8192 x 28672 86.6 against 82.8, 64 x 8192 x 16384
+  // 55.0 against 53.0, 64 x 16384 x 8192 53.5 against 51.6, and from an unsplit 128-column grid 64 x 28672 x
+  // 8192 86.0 against 82.9 (33 rows 79.5 against 80.7).  The line at K / (4 * splits) >= 512 is the one of 17 to
+  // 32 rows; just below it 64 x 8192 x 8192 and 64 x 8192 x 12288 run within 2% either way, while 256 columns
+  // would be the faster form at 64 x 12288 x 8192 (41.6 against 46.9) and of grids past 256 strips (64 x 49152 x
+  // 4096 68.2 against 86.1).
   if (!p.ws_absent && !b_unaligned && (splits >= 2 || mr == 4) && p.K >= 8192) {
     const int strips2 = (p.N + 255) / 256, splits2 = splits_for(256, strips2);
     if (splits2 >= 2 && strips2 * splits2 >= strips * splits && p.K / (4 * splits2) >= (mr == 1 ? 256 : 512))
@@ -604,8 +605,9 @@ int skinny_columns(const GemmProblem& p) { return stream_shape(p).splits ? strea
 // More 128-column strips than CUs, on B rows that are not 16-byte aligned or with rounds less than
 // 2/3 filled on average: the tile kernels run the problem faster.  Measured (B rotating through
 // HBM, auto-picked tiles against the streaming kernel): unaligned 16 x 33001 x 8192 129 us against
-// 207.6, 16 x 50257 x 4096 92.0 against 140.7, 64 x 50257 x 4096 100.3 against 155.9; aligned
-// 16 x 33000 x 8192 (258 strips) 118.1 against 140.1, 16 x 40000 x 8192 (313) 121.8 against 128.2.
+// 207.6, 16 x 50257 x 4096 92.0 against 140.7, 64 x 50257 x 4096 86.0 against 99.1; aligned
+// 16 x 33000 x 8192 (258 strips) 118.1 against 140.1, 16 x 40000 x 8192 (313) 121.8 against 128.2, 64 x
+// 33000 x 8192 127.4 against 157.5 (64 x 40000 x 8192 145.2 against 139.0).
 // Fuller rounds stream faster: 16 x 49152 x 8192 (384 strips) 150.4 against 172.1, 32 x 81920 x
 // 4096 (640) 134.9 against 151.0, 16 x 151936 x 4096 (1187) 204.2 against 233.3, 16 x 65536 x
 // 8192 174.4 against 186.7 (16 x 100000 x 4096, 782 strips: 184.9 streamed, 163.0 on tiles).
@@ -613,7 +615,7 @@ int skinny_columns(const GemmProblem& p) { return stream_shape(p).splits ? strea
 // threshold rises to 1.8 (measured: 16 x 33000 x 8192, 1.98, tiles 130.2 against 165.5 streamed;
 // 16 x 40000 x 8192, 1.64, tiles 129.4 against 123.3-125.2 streamed); unaligned rows still go to
 // tiles (16 x 33001 x 8192 147.2 against 201.6; 16 x 50257 x 4096 96.0 against 126.9-130.2;
-// 64 x 50257 x 4096 97.2 against 152.0).
+// 64 x 50257 x 4096 86.7 against 99.2).
 bool skinny_prefers_tiles(const GemmProblem& p) {
   const StreamShape sh = stream_shape(p);
   if (sh.splits == 0) return false;  // the wave-split kernel
@@ -626,11 +628,11 @@ bool skinny_prefers_tiles(const GemmProblem& p) {
 
 // 33 to 64 rows on a 128-column grid of 2 or 3 K splits with K <= 4096 (many strips, short
 // streams): the 64 x 64 tile kernel, whose B panels the M <= 64 rows share, runs them faster.
-// Measured (B rotating through HBM, whole calls): 64 x 14336 x 4096 225.1 against 214.4 TFLOP/s
-// streamed, 64 x 16384 x 4096 264.2 against 236.0, 64 x 11008 x 4096 190.5 against 180.8,
-// 56 x 14336 x 4096 200.7 against 191.4, 48 x 14336 x 4096 174.3 against 166.7, 40 x 11008 x
-// 4096 124.9 against 121.9.  At K = 8192 the same grids stream faster than the tile picked for
-// them (64 x 10240 x 8192: 249.7 streamed, 175 on 64 x 64 tiles).
+// Measured (B rotating through HBM, whole calls, us, 64 x 64 tiles against streamed): 64 x 11008 x 2048
+// 11.1 against 15.5, 64 x 14336 x 3000 22.2 against 24.2, 33 x 14336 x 3000 17.4 against 22.3, 64 x 16384 x 4096
+// 30.4 against 32.2, 64 x 11008 x 4096 23.6 against 23.8.  K = 4096 is where the two cross: 12288 and 14336
+// columns stream faster there (64 rows 28.1 against 30.1 and 29.8 against 31.3).  At K = 8192 the same grids
+// stream (64 x 12288 x 8192 46.9 against 59.3).
 bool skinny_tiles_faster(const GemmProblem& p) {
   const StreamShape sh = stream_shape(p);
   return !p.ws_absent && sh.mr == 4 && sh.ns == 128 && sh.splits >= 2 && sh.splits <= 3 && p.K <= 4096;
@@ -662,7 +664,7 @@ bool skinny_ok(const GemmProblem& p) {
 
 // B operands this large are streamed with non-temporal loads.  Measured on MI355X (interleaved,
 // three B buffers rotating): 16 x 8192 x 8192 32.9 -> 30.8 us per call, 32 x 8192 x 8192 34.8 ->
-// 32.7, 64 x 14336 x 4096 (112 MiB) 36.6 -> 35.4; with 64 MiB of B (16 x 4096 x 8192: three
+// 32.7; with 64 MiB of B (16 x 4096 x 8192: three
 // buffers fit the 256 MB Infinity Cache) 17.5 -> 18.4, slower, so smaller B keeps cached loads.
 // The in-workgroup kernel's 64-byte strips ran 30-40% slower with them (not used there).
 constexpr int64_t kNtStreamBytes = 96ll << 20;
