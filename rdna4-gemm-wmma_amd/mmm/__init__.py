@@ -243,25 +243,23 @@ def _workspace(device, st: C.c_void_p, nbytes: int):
         return t
 
 
-def _ws_of(t):
-    return (None, 0) if t is None else (C.c_void_p(t.data_ptr()), t.numel() * t.element_size())
-
-
-def _ws_args(workspace, device, st, need):
+def _ws_args(workspace, device, st, need, *args):
     """(tensor, pointer, bytes) for a call: the caller's tensor, none (workspace=False), the per-stream
-    cache's, or under graph capture one of need() bytes of the graph's own (at least 16: with a
+    cache's, or under graph capture one of need(*args) bytes of the graph's own (at least 16: with a
     workspace the library may choose another unsplit kernel than without).  The caller keeps the
     tensor until its launch has been enqueued."""
     if workspace is False:
         return None, None, 0
     t = workspace
     if t is None:
-        capture = _capture_id(st)
+        capture = _capture_id(st) if st.value else None
         if capture is None:
             t = _workspace(device, st, MAX_WORKSPACE_BYTES)
         else:
-            t = _graph_workspace(device, st, capture, max(need(), 16))
-    return t, *_ws_of(t)
+            t = _graph_workspace(device, st, capture, max(need(*args), 16))
+            if t is None:
+                return None, None, 0
+    return t, C.c_void_p(t.data_ptr()), t.numel() * t.element_size()
 
 
 def gemm(A, B, C_out=None, tile=None, stream=None, workspace=None):
@@ -293,12 +291,12 @@ def gemm(A, B, C_out=None, tile=None, stream=None, workspace=None):
     L = lib()
     if tile is None:
         # one library call: the per-stream workspace holds the largest split the library plans
-        ws, wp, wb = _ws_args(workspace, A.device, st, lambda: _gemm_need(A, B, C_out, M, N, K, lda, ldb, ldc))
+        ws, wp, wb = _ws_args(workspace, A.device, st, _gemm_need, A, B, C_out, M, N, K, lda, ldb, ldc)
         rc = L.mmm_gemm_f16f32_ws(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, wp, wb, st)
         _check("mmm_gemm_f16f32_ws", rc)
     else:
         params = TILES[tile] if isinstance(tile, str) else tuple(tile)
-        ws, wp, wb = _ws_args(workspace, A.device, st, lambda: MAX_WORKSPACE_BYTES)
+        ws, wp, wb = _ws_args(workspace, A.device, st, int, MAX_WORKSPACE_BYTES)
         rc = L.mmm_gemm_f16f32_tiled(_ptr(A), _ptr(B), _ptr(C_out), M, N, K, lda, ldb, ldc, *params, wp, wb, st)
         _check("mmm_gemm_f16f32_tiled", rc)
     return C_out
@@ -312,6 +310,10 @@ def _bound(fn, name: str, args: tuple, keep: tuple):
 
     launch.tensors = keep  # the launcher holds its operands (and workspace) alive
     return launch
+
+
+def _ws_of(t):
+    return (None, 0) if t is None else (C.c_void_p(t.data_ptr()), t.numel() * t.element_size())
 
 
 def _bound_ws(fn, name: str, args, workspace, device, st, need, keep: tuple):
@@ -516,7 +518,7 @@ def contract(desc: ContractDesc, A, B, C_out, stream=None, workspace=None):
         raise TypeError("C must be a CUDA float32 tensor")
     st = _stream(stream)
     L = lib()
-    ws, wp, wb = _ws_args(workspace, A.device, st, lambda: _contract_need(desc, A, B, C_out))
+    ws, wp, wb = _ws_args(workspace, A.device, st, _contract_need, desc, A, B, C_out)
     rc = L.mmm_contract5d_f16f32_ws(C.byref(desc), _ptr(A), _ptr(B), _ptr(C_out), wp, wb, st)
     _check("mmm_contract5d_f16f32_ws", rc)
     return C_out
